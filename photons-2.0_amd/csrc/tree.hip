@@ -742,7 +742,7 @@ __global__ void __launch_bounds__(kSubThreads) k_subtree(DevSizes *sz, int level
 {
     constexpr int W = kSubThreads / kWave, NL = kSubNodes + 1;
     __shared__ double sx[kSubtree], sy[kSubtree], sz_[kSubtree], nsplit[kSubNodes];
-    __shared__ int sidx[kSubtree], s_base, s_nn, s_nl, s_fail;
+    __shared__ int sidx[kSubtree], s_base, s_nn, s_nl, s_fail, s_stop;
     __shared__ uint16_t perm[2][kSubtree];
     __shared__ uint16_t nstart[kSubNodes], ncount[kSubNodes], nsize[kSubNodes], nlsize[kSubNodes], ndfs[kSubNodes],
         nlf[kSubNodes];
@@ -751,9 +751,13 @@ __global__ void __launch_bounds__(kSubThreads) k_subtree(DevSizes *sz, int level
     __shared__ uint16_t lstart[NL], lcount[NL], ldfs[NL], lnum[NL];
     __shared__ int16_t lparent[NL];
     __shared__ uint16_t lev[kMaxDepth + 2];
-    if (sz->overflow) return;
     const int l = blockIdx.x;
     if (l >= sz->ldo[levels + 1]) return;
+    // other workgroups set the overflow bits meanwhile: one thread looks at them for all, so
+    // that no wavefront stays behind with what the others would have set up
+    if (threadIdx.x == 0) s_stop = __hip_atomic_load(&sz->overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_stop) return;
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int m = T.l_count[l], base = T.l_start[l], depth = depth_of(l_depth[l]);
     const Particles S = (depth & 1) ? B : A;  // particles of depth D are in buffer D % 2
