@@ -503,6 +503,12 @@ int photons_force_device_static(photons_ctx *x, int64_t n, const double *d_pos, 
         // the context as it was (buffers, counts, lists): restored afterwards, so its last
         // ordinary evaluation stays inspectable
         const Ctx kept = c;
+        // but for the pair tables, which stay as this evaluation leaves them on the device
+        auto restore = [&] {
+            const PairTab now[2] = {c.pair_tab[0], c.pair_tab[1]};
+            c = kept;
+            for (int k = 0; k < 2; k++) c.pair_tab[k] = now[k];
+        };
         c.n = n;
         for (DevBuf *b : eval_bufs(c)) *b = DevBuf();
         c.tcap = c.lcap = 0;
@@ -516,13 +522,13 @@ int photons_force_device_static(photons_ctx *x, int64_t n, const double *d_pos, 
         } catch (...) {
             g_arena = nullptr;
             (void)hipStreamSynchronize(c.stream);
-            c = kept;
+            restore();
             throw;
         }
         g_arena = nullptr;
         double ph[16];
         std::memcpy(ph, c.phase_ms, sizeof ph);
-        c = kept;
+        restore();
         std::memcpy(c.phase_ms, ph, sizeof ph);
         return 0;
     } catch (const std::exception &e) {
