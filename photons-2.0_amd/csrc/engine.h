@@ -76,6 +76,7 @@ struct DevSizes {
     int lvl[kMaxLevels + 1];          // first temporary node of depth d
     int ldo[kMaxLevels + 1];          // first temporary leaf of depth d
     int lv_nodes, lv_leaves, lv_done;  // a level being split: nodes, leaves handed out, segments finished
+    int lv_large;                      // its children's most particles, where that is many
     int tmp_cells, sub_nodes, sub_leaves;  // cells of the subtrees built so far
 };
 
@@ -98,7 +99,8 @@ struct Plan {
     int scap = 0;          // nodes of one level
     int tcap = 0, lcap = 0;  // nodes, leaves
     bool subtrees = false;   // the tree is built by subtrees: levels, scap, top and stems
-    int top = 0, stems = 0;  // are those of the top tree (its nodes; its leaves, the stems)
+    int top = 0, stems = 0;  // are those of the top tree (its nodes; its leaves, the stems),
+    int chunked = 0;         // whose leading levels go by chunks
     int64_t dl_cap = 0;    // down list entries
     int64_t p2p_cap = 0, m2l_cap = 0;  // list entries
     int item_cap = 0;      // M2L work items
@@ -121,7 +123,7 @@ struct Reuse {
 struct Measure {
     int levels = 0, scap = 0, ntmp = 0, nleaf = 0, depths = 0, items = 0;
     bool subtrees = false;
-    int top = 0, stems = 0, tree_depth = 0;
+    int top = 0, stems = 0, chunked = 0, tree_depth = 0;
     int64_t dl = 0, p2p = 0, m2l = 0;
 };
 

@@ -554,6 +554,7 @@ static void plan_from_measure(Ctx &c, double margin)
     p.subtrees = m.subtrees;
     p.top = (int)up(m.top, 64);
     p.stems = (int)up(m.stems, 64);
+    p.chunked = m.chunked;
     p.scap = (int)up(m.scap, 64);
     p.tcap = (int)up(m.ntmp, 1024);
     p.lcap = (int)up(m.nleaf, 1024);

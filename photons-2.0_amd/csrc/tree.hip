@@ -160,9 +160,10 @@ __global__ void __launch_bounds__(256) k_chunk_count(LevelArgs a, const double *
 
 // per segment: particles left of the split, the degenerate-partition flag, and the kinds
 // of its two children (new nodes in the high 32 bits, new leaves in the low 32 bits, packed
-// so that one scan gives both offsets; the leaf count stays below 2^32, so no carry crosses)
+// so that one scan gives both offsets; the leaf count stays below 2^32, so no carry crosses);
+// *large: the most particles of a child that holds more than `over`
 __global__ void k_seg_counts(LevelArgs a, const int *__restrict__ rpre, int maxleaf, int *__restrict__ nleft,
-                             int *__restrict__ flag, uint64_t *__restrict__ kinds)
+                             int *__restrict__ flag, uint64_t *__restrict__ kinds, int over, int *large)
 {
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int S = a.nseg(), seg0 = a.seg0();
@@ -186,6 +187,7 @@ __global__ void k_seg_counts(LevelArgs a, const int *__restrict__ rpre, int maxl
     }
     nleft[s] = nl;
     flag[s] = f;
+    if (max(nl, ct - nl) > over) atomicMax(large, max(nl, ct - nl));
     const int k = (nl > maxleaf) + (ct - nl > maxleaf);
     kinds[s] = ((uint64_t)k << 32) | (uint64_t)(2 - k);
 }
@@ -328,6 +330,7 @@ __global__ void k_level_step(DevSizes *sz, int d, const uint64_t *__restrict__ k
     const int S = sz->lvl[d + 1] - sz->lvl[d];
     const uint64_t tot = kind_off[S];
     const int nn = (int)(tot >> 32), nl = (int)(uint32_t)tot;
+    sz->lv_large = 0;
     int ovf = 0;
     if ((int64_t)sz->lvl[d + 1] + nn > tcap) ovf |= kOvfNodes;
     if (nn > scap) ovf |= kOvfNodes;
@@ -349,7 +352,7 @@ __global__ void k_tree_roots(int nbox, const int64_t *__restrict__ box_off, cons
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b == 0) {
         sz->overflow = 0;
-        sz->lv_nodes = sz->lv_leaves = sz->lv_done = 0;
+        sz->lv_nodes = sz->lv_leaves = sz->lv_done = sz->lv_large = 0;
         sz->tmp_cells = sz->sub_nodes = sz->sub_leaves = sz->maxdepth = 0;
         sz->lvl[0] = 0;
         sz->lvl[1] = nbox;
@@ -554,7 +557,16 @@ __global__ void k_emit_leaves(const DevSizes *__restrict__ sz, const int *__rest
 constexpr int kSubtree = 1024;     // particles of a stem, at leaves of 8 and more
 constexpr int kSubNodes = 512;     // nodes of a subtree (leaves: one more)
 constexpr int kSubThreads = 512;
-constexpr int64_t kWgSegment = 32768;
+// Segments that one workgroup splits: a level goes by chunks of all its segments while any
+// holds more.  A mean split leaves most of a concentrated box in one segment for several
+// levels, so that the largest segment counts and not the level.  Tree phase, by the level's
+// number against this: 2M particles with half of them in one clump 2.7 -> 1.2 ms (all levels by
+// chunks: 1.6), 2M with log-uniform radii over six decades 3.5 -> 1.3 (1.8), 256^3 clustered
+// ones 8.3 -> 7.1 (9.2).  A workgroup takes 2.1 us per 1000 particles, a level by chunks some 50 us and 0.25
+// ms at 256^3: limits of 8192, 16384, 32768, 65536 and 131072 give 6.5, 6.9, 7.4, 7.6 and 8.1 ms
+// there, 1.25, 1.25, 1.32, 1.42 and 1.57 at 128^3; replayed evaluations of 20,000 to 100,000
+// particles are within 1% from 12288 to 32768.
+constexpr int kWgSegment = 24576;
 
 // stems by leaf size: few enough particles that the nodes fit
 static inline int subtree_particles(int maxleaf) { return maxleaf >= 8 ? kSubtree : maxleaf >= 4 ? 512 : 256; }
@@ -565,7 +577,7 @@ static inline int subtree_particles(int maxleaf) { return maxleaf >= 8 ? kSubtre
 // it).  The last workgroup writes the next level's ranges.
 __global__ void __launch_bounds__(1024) k_split_level(DevSizes *sz, int d, TreeTmp T, int *__restrict__ l_depth,
                                                       int stop, int node_cap, int leaf_cap, int scap, Particles src,
-                                                      Particles dst, double *__restrict__ partial)
+                                                      Particles dst)
 {
     constexpr int W = 1024 / kWave;
     __shared__ int wcnt[W];
@@ -581,32 +593,33 @@ __global__ void __launch_bounds__(1024) k_split_level(DevSizes *sz, int d, TreeT
     }
     const int v = seg0 + s, st = T.t_start[v], ct = T.t_count[v], axis = d % 3;
     const double *coord = axis == 0 ? src.x : (axis == 1 ? src.y : src.z);
-    // the mean: a partial per chunk, combined by one wavefront (k_chunk_sum, k_mean); those of
-    // a large segment at (start / 1024) + chunk, apart from the other segments' of the level
+    // the mean: a partial per chunk, combined by one wavefront (k_chunk_sum, k_mean), 64 chunks
+    // at a time
     const int nch = (ct + kChunk - 1) / kChunk;
-    double *const part = nch <= kWave ? s_part : partial + st / (kChunk / 2);
-    for (int c = wave; c < nch; c += W) {
-        const int b = st + c * kChunk, e = min(b + kChunk, st + ct);
-        double x = 0.0;
-        int i = b + lane;
-        for (; i + 3 * kWave < e; i += 4 * kWave) {
-            const double x0 = coord[i], x1 = coord[i + kWave], x2 = coord[i + 2 * kWave], x3 = coord[i + 3 * kWave];
-            x += x0;
-            x += x1;
-            x += x2;
-            x += x3;
+    double mean = 0.0;
+    for (int c0 = 0; c0 < nch; c0 += kWave) {
+        if (c0 > 0) __syncthreads();  // the last ones are read
+        for (int c = c0 + wave; c < min(c0 + kWave, nch); c += W) {
+            const int b = st + c * kChunk, e = min(b + kChunk, st + ct);
+            double x = 0.0;
+            int i = b + lane;
+            for (; i + 3 * kWave < e; i += 4 * kWave) {
+                const double x0 = coord[i], x1 = coord[i + kWave], x2 = coord[i + 2 * kWave], x3 = coord[i + 3 * kWave];
+                x += x0;
+                x += x1;
+                x += x2;
+                x += x3;
+            }
+            for (; i < e; i += kWave) x += coord[i];
+            x = wave_sum(x);
+            if (lane == 0) s_part[c - c0] = x;
         }
-        for (; i < e; i += kWave) x += coord[i];
-        x = wave_sum(x);
-        if (lane == 0) part[c] = x;
+        __syncthreads();
+        if (wave == 0 && c0 + lane < nch) mean += s_part[lane];
     }
-    __threadfence_block();
-    __syncthreads();
     if (wave == 0) {
-        double x = 0.0;
-        for (int c = lane; c < nch; c += kWave) x += part[c];
-        x = wave_sum(x);
-        if (lane == 0) s_split = x / (double)ct;
+        mean = wave_sum(mean);
+        if (lane == 0) s_split = mean / (double)ct;
     }
     __syncthreads();
     const double split = s_split;
@@ -1244,12 +1257,12 @@ bool build_tree(Ctx &c)
     std::vector<int> lvl = {0, nbox};  // host copies of the level ranges (ordinary evaluation)
     std::vector<int> ldo = {0, 0};
     const int cextra = (int)((n + kChunk - 1) / kChunk);
-    // a level's segments by a workgroup each, once they are down to kWgSegment particles
-    // when all are alike (a larger one takes its workgroup longer); a forest's boxes start
-    // with its largest
-    int64_t nmax = 0;
-    for (int b = 0; b < nbox; b++) nmax = std::max(nmax, c.box_off[b + 1] - c.box_off[b]);
-    double *wg_part = sub ? tree_buf<double>(c, c.chunk_part, n / (kChunk / 2) + 2 + (size_t)cextra, "tree level") : nullptr;
+    // levels by chunks while a segment holds more than this, then by a workgroup per segment
+    // (a planned evaluation: as many as in the one it was measured from)
+    const int wg_segment = sub ? kWgSegment : INT32_MAX;
+    int64_t largest = 0;  // segment of the level, 0 once there are none above wg_segment
+    for (int b = 0; b < nbox; b++) largest = std::max(largest, c.box_off[b + 1] - c.box_off[b]);
+    int chunked = 0;      // levels by chunks
     int depth = 0;
     for (;; depth++) {
         int Scap;
@@ -1262,7 +1275,7 @@ bool build_tree(Ctx &c)
             Scap = lvl[depth + 1] - lvl[depth];
         }
         const int axis = depth % 3;
-        if (sub && (depth >= 40 || (nmax >> depth) <= kWgSegment)) {
+        if (sub && (planned ? depth >= c.plan.chunked : largest <= wg_segment)) {
             if (!planned) {  // room for two children of every segment
                 const int ntmp = lvl[depth + 1], nleaf = ldo[depth + 1];
                 if (ntmp + 2 * Scap > T.tcap) alloc_nodes(std::max(2 * T.tcap, ntmp + 2 * Scap), T.tcap);
@@ -1270,7 +1283,7 @@ bool build_tree(Ctx &c)
             }
             k_split_level<<<Scap, 1024, 0, st>>>(sz, depth, T, l_depth, stop, planned ? want_nodes : T.tcap,
                                                  planned ? want_leaves : T.lcap, planned ? c.plan.scap : INT32_MAX, A,
-                                                 B, wg_part);
+                                                 B);
             std::swap(A, B);
             if (!planned) {
                 PH_CHECK(hipMemcpyAsync(pin, &sz->lvl[depth + 2], sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1281,6 +1294,7 @@ bool build_tree(Ctx &c)
             }
             continue;
         }
+        chunked = depth + 1;
         // sum over segments of ceil(count / kChunk) <= S + ceil(n / kChunk)
         const int C = Scap + cextra;
         int *seg_chunk = tree_buf<int>(c, c.seg_chunk, Scap + 1, "tree level");
@@ -1301,10 +1315,11 @@ bool build_tree(Ctx &c)
         k_mean<<<blocks(Scap, kWavesPerBlock), 256, 0, st>>>(a, partial, T.t_split);
         k_chunk_count<<<blocks(C + 1, kWavesPerBlock), 256, 0, st>>>(a, T.t_split, rcnt);
         exclusive_scan(c, rcnt, rpre, C + 1);
-        k_seg_counts<<<blocks(Scap + 1, 256), 256, 0, st>>>(a, rpre, stop, nleft, flag, kinds);
+        k_seg_counts<<<blocks(Scap + 1, 256), 256, 0, st>>>(a, rpre, stop, nleft, flag, kinds, wg_segment, &sz->lv_large);
         exclusive_scan_u64(c, kinds, kind_off, Scap + 1);
         if (!planned) {
             PH_CHECK(hipMemcpyAsync(pin, kind_off + Scap, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+            PH_CHECK(hipMemcpyAsync(pin + 2, &sz->lv_large, sizeof(int), hipMemcpyDeviceToHost, st));
             PH_CHECK(hipEventRecord(c.counts_ready, st));
         }
         // the partition runs while the host reads the counts
@@ -1324,6 +1339,7 @@ bool build_tree(Ctx &c)
             if (nleaf + new_leaves > T.lcap) alloc_leaves(std::max(2 * T.lcap, nleaf + new_leaves + 1024), T.lcap);
             lvl.push_back(ntmp + new_nodes);
             ldo.push_back(nleaf + new_leaves);
+            largest = pin[2];
         }
         k_make_children<<<blocks(Scap, 256), 256, 0, st>>>(a, T, axis, stop, nleft, kind_off, l_depth);
         // the planned capacities (the arrays may be larger, from earlier evaluations)
@@ -1379,6 +1395,7 @@ bool build_tree(Ctx &c)
             Measure &m = c.meas;
             m.subtrees = true;
             m.levels = levels;
+            m.chunked = chunked;
             m.top = lvl[levels];
             m.stems = ldo[levels + 1];
             m.ntmp = c.nnode;
