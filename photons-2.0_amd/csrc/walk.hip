@@ -377,6 +377,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(EU
     const int nheavy = a.heavy_only ? a.st->heavy[slot][STORE] : 0;
     const int x0 = (int)(blockIdx.x % kXcds);
     if (STORE && tid < 2 * kOut) w.held[tid / 2][tid % 2] = a.st->chunk[blockIdx.x][tid / 2][tid % 2];
+    wave_sync();  // (thread 0 reads them)
     uint64_t total[kOut] = {};  // thread 0's
     for (int i = (int)(blockIdx.x / kXcds);; i += (int)(gridDim.x / kXcds)) {
         int u;
