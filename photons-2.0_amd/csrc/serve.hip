@@ -41,9 +41,10 @@ namespace {
         if (e_ != hipSuccess) throw std::runtime_error(std::string(#x) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-// evaluation buffers per particle of a batch: tree, expansions, lists (~37 entries
-// per particle at the 256^3 density, 8 bytes each plus sort buffers) and the
-// batch's own pos/acc copies, rounded up
+// evaluation buffers per particle of a batch: tree, expansions, lists, the P2P slices' parts
+// and the batch's own pos/acc copies.  Contexts of 64 clustered boxes of 64^3 particles hold 511
+// (FP32-mixed) and 729 bytes (FP64) a particle at leaves of 32 and p = 4, 842 with boxes of
+// 32^3; leaves of 16 at p = 5 take 1405 and 1648
 constexpr double kTransientBytesPerParticle = 1024.0;
 constexpr double kResidentBytesPerParticle = 72.0;  // pos, vel, acc (3 doubles each)
 constexpr int kLaneMeshes = 8;                      // PM contexts kept per lane
