@@ -118,12 +118,14 @@ int photons_force_boxes_device(photons_ctx *ctx, int nbox, const int64_t *counts
 int photons_force_device_static(photons_ctx *ctx, int64_t n, const double *d_pos, double *d_acc);
 
 /* Tuning (no counterpart in the reference, which takes MAXLEAF from its parameter
- * file, src/initial.c:172-173, untuned).  The FP32-mixed P2P kernel stages 256 or
- * 512 source particles per batch in LDS (default 256).  photons_autotune_boxes times leaf
- * sizes 16/32/64 x staging 256/512 (staging only for FP32-mixed) on the
- * caller's batch, keeps the fastest in the context and leaves its result in
- * d_acc; ms[6] (or NULL) gets the mean ms per evaluation of each candidate,
- * leaf-major, -1 where a candidate was skipped (boxes of <= leaf particles). */
+ * file, src/initial.c:172-173, untuned).  The P2P kernel of FP32-mixed boxes of fewer
+ * than 900,000 particles (and of softenings below some 4e-4 rs) stages 256 or 512
+ * source particles per batch in LDS (default 256); the other P2P kernels have no such
+ * choice.  photons_autotune_boxes times leaf sizes 16/32/64, by staging 256/512 where a
+ * box takes that kernel, on the caller's batch, keeps the fastest in the context and
+ * leaves its result in d_acc; ms[6] (or NULL) gets the mean ms per evaluation of each
+ * candidate, leaf-major, -1 where a candidate was skipped (boxes of <= leaf particles;
+ * a staging size that changes nothing). */
 int photons_set_p2p_stage(photons_ctx *ctx, int stage);
 int photons_get_p2p_stage(const photons_ctx *ctx);
 int photons_autotune_boxes(photons_ctx *ctx, int nbox, const int64_t *counts, const double *lengths,

@@ -285,6 +285,7 @@ void downward_pass(Ctx &c);              // L2L
 void p2p_l2p_pass(Ctx &c, bool with_l2p, bool accumulate);  // acc (+)= P2P (+ L2P)
 
 size_t pair_table_bytes(bool f32);  // of the largest pair table
+bool p2p_staged(const Ctx &c, int nbox, const int64_t *counts);  // a box takes the FP32 kernel that stages batches
 
 int nterms_of(int order);
 void phase_mark(Ctx &c);                 // records a timing event (when enabled)

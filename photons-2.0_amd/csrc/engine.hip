@@ -761,8 +761,8 @@ int photons_set_p2p_stage(photons_ctx *x, int stage)
 
 int photons_get_p2p_stage(const photons_ctx *x) { return x->c.p2p_stage; }
 
-// Leaf size (16, 32, 64) and, for FP32-mixed, the P2P staging size (256, 512) timed
-// on the caller's own batch: each candidate runs reps + 1 evaluations (the first
+// Leaf size (16, 32, 64) and, where a box takes the P2P kernel that has one, the staging
+// size (256, 512) timed on the caller's own batch: each candidate runs reps + 1 evaluations (the first
 // untimed), wall clock from queueing to the end of the last one; the fastest is
 // kept in the context and d_acc holds its result.
 int photons_autotune_boxes(photons_ctx *x, int nbox, const int64_t *counts, const double *lengths,
@@ -777,12 +777,14 @@ int photons_autotune_boxes(photons_ctx *x, int nbox, const int64_t *counts, cons
         const int keep_stage = c.p2p_stage;
         const int leaves[3] = {16, 32, 64}, stages[2] = {256, 512};
         const bool f32 = c.prm.precision == PHOTONS_FP32_MIXED;
+        const bool staged = f32 && nbox > 0 && counts && p2p_staged(c, nbox, counts);
         double best = 1e300;
         int bl = keep.maxleaf, bs = c.p2p_stage;
         for (int i = 0; i < 3; i++)
             for (int j = 0; j < 2; j++) {
                 if (ms) ms[2 * i + j] = -1.0;
                 if (!f32 && j == 0) continue;  // the staging size is an FP32 choice
+                if (f32 && !staged && stages[j] != keep_stage) continue;  // it would change nothing
                 c.prm.maxleaf = leaves[i];
                 c.p2p_stage = stages[j];
                 if (!check_boxes(c, nbox, counts, lengths).empty()) continue;  // boxes too small for this leaf
