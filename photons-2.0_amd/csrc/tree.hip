@@ -452,21 +452,55 @@ __global__ void k_number(const int *__restrict__ t_son, const DevSizes *__restri
 }
 
 // the roots (temporary ids 0 .. nbox-1, one per box, in box order) take consecutive
-// depth-first ranges: dfs and lfirst of root b = cells and leaves of the earlier roots
-__global__ void k_root_starts(int nbox, const DevSizes *__restrict__ sz, const int *__restrict__ size,
-                              const int *__restrict__ lsize, int *__restrict__ dfs, int *__restrict__ lfirst,
-                              int *__restrict__ box_root)
+// depth-first ranges: dfs and lfirst of root b = cells and leaves of the earlier roots.
+// By one workgroup of 1024 threads, K consecutive boxes each (5,000 boxes by one thread took
+// 380 us)
+__device__ void number_roots(int nbox, int nleaf, const int *size, const int *lsize, int *dfs, int *lfirst,
+                             int *box_root)
 {
-    if (blockIdx.x != 0 || threadIdx.x != 0 || sz->overflow) return;
-    const int nleaf = sz->nleaf;
-    int d = 0, lf = 0;
-    for (int b = 0; b < nbox; b++) {
+    constexpr int W = 1024 / kWave;
+    __shared__ int s_cells[W], s_leaves[W];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int K = (nbox + 1023) / 1024, b0 = min((int)threadIdx.x * K, nbox), b1 = min(b0 + K, nbox);
+    int cells = 0, leaves = 0;
+    for (int b = b0; b < b1; b++) {
+        cells += size[b];
+        leaves += lsize[b];
+    }
+    int d = cells, lf = leaves;  // inclusive sums
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int x = __shfl_up(d, o, kWave), y = __shfl_up(lf, o, kWave);
+        if (lane >= o) {
+            d += x;
+            lf += y;
+        }
+    }
+    if (lane == kWave - 1) {
+        s_cells[wave] = d;
+        s_leaves[wave] = lf;
+    }
+    __syncthreads();
+    d -= cells;
+    lf -= leaves;
+    for (int w = 0; w < wave; w++) {
+        d += s_cells[w];
+        lf += s_leaves[w];
+    }
+    for (int b = b0; b < b1; b++) {
+        const int c = size[b], l = lsize[b];
         dfs[b] = d;
         lfirst[b] = lf;
         box_root[b] = nleaf + d - lf;
-        d += size[b];
-        lf += lsize[b];
+        d += c;
+        lf += l;
     }
+}
+
+__global__ void __launch_bounds__(1024) k_root_starts(int nbox, const DevSizes *__restrict__ sz, const int *size,
+                                                      const int *lsize, int *dfs, int *lfirst, int *box_root)
+{
+    if (!sz->overflow) number_roots(nbox, sz->nleaf, size, lsize, dfs, lfirst, box_root);
 }
 
 
@@ -567,6 +601,14 @@ constexpr int kSubThreads = 512;
 // there, 1.25, 1.25, 1.32, 1.42 and 1.57 at 128^3; replayed evaluations of 20,000 to 100,000
 // particles are within 1% from 12288 to 32768.
 constexpr int kWgSegment = 24576;
+
+// Forests of more than kManyBoxes boxes of at most kFewLeaves leaves' worth of particles go
+// level by level: there are few levels, whereas each box costs its subtrees' workgroups some
+// 0.13 us.  Tree phase by subtrees and by levels, leaves of 32: 100,000 boxes of 40 particles
+// 13.3 and 1.04 ms, 5,000 of 64 0.65 and 0.21, 16,000 of 250 2.28 and 0.87, 8,000 of 500 1.17
+// and 0.94, 4,000 of 1000 0.68 and 1.02; 2,133 of 150 0.29 and 0.29, 800 of 100 0.14 and 0.26.
+// Leaves of 8: 5,000 of 64 0.62 and 0.46, 16,000 of 250 2.5 and 2.9.
+constexpr int kManyBoxes = 2048, kFewLeaves = 16;
 
 // stems by leaf size: few enough particles that the nodes fit
 static inline int subtree_particles(int maxleaf) { return maxleaf >= 8 ? kSubtree : maxleaf >= 4 ? 512 : 256; }
@@ -1044,17 +1086,7 @@ __global__ void __launch_bounds__(1024) k_top_number(DevSizes *sz, int levels, c
         __threadfence_block();
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const int nleaf = sz->nleaf;
-        int d = 0, lf = 0;
-        for (int b = 0; b < nbox; b++) {
-            dfs[b] = d;
-            lfirst[b] = lf;
-            box_root[b] = nleaf + d - lf;
-            d += size[b];
-            lf += lsize[b];
-        }
-    }
+    number_roots(nbox, sz->nleaf, size, lsize, dfs, lfirst, box_root);
     __threadfence_block();
     __syncthreads();
     for (int d = 0; d < levels; d++) {
@@ -1193,7 +1225,10 @@ bool build_tree(Ctx &c)
     const bool planned = c.plan.active;
     const int64_t n = c.n;
     const int maxleaf = c.prm.maxleaf;
-    const bool sub = planned ? c.plan.subtrees : !c.no_subtrees;
+    int64_t nmax = 0;
+    for (int b = 0; b < c.nbox; b++) nmax = std::max(nmax, c.box_off[b + 1] - c.box_off[b]);
+    const bool few_levels = c.nbox > kManyBoxes && nmax <= (int64_t)kFewLeaves * maxleaf;
+    const bool sub = planned ? c.plan.subtrees : !c.no_subtrees && !few_levels;
     const int stop = sub ? std::max(maxleaf, subtree_particles(maxleaf)) : maxleaf;  // segments no longer split here
     hipStream_t st = c.stream;
     DevSizes *sz = dptr<DevSizes>(c.sizes);
@@ -1260,8 +1295,7 @@ bool build_tree(Ctx &c)
     // levels by chunks while a segment holds more than this, then by a workgroup per segment
     // (a planned evaluation: as many as in the one it was measured from)
     const int wg_segment = sub ? kWgSegment : INT32_MAX;
-    int64_t largest = 0;  // segment of the level, 0 once there are none above wg_segment
-    for (int b = 0; b < nbox; b++) largest = std::max(largest, c.box_off[b + 1] - c.box_off[b]);
+    int64_t largest = nmax;  // segment of the level, 0 once there are none above wg_segment
     int chunked = 0;      // levels by chunks
     int depth = 0;
     for (;; depth++) {
@@ -1439,7 +1473,7 @@ bool build_tree(Ctx &c)
     for (int d = levels - 1; d >= 0; d--)
         k_sizes<<<blocks(level_bound(d), 256), 256, 0, st>>>(T.t_son, sz, d, size, lsize);
     int *box_root = tree_buf<int>(c, c.d_box_root, nbox, "box roots");
-    k_root_starts<<<1, 1, 0, st>>>(nbox, sz, size, lsize, dfs, lfirst, box_root);
+    k_root_starts<<<1, 1024, 0, st>>>(nbox, sz, size, lsize, dfs, lfirst, box_root);
     for (int d = 0; d < levels; d++)
         k_number<<<blocks(level_bound(d), 256), 256, 0, st>>>(T.t_son, sz, d, size, lsize, dfs, lfirst, l_final,
                                                               l_dfs);
