@@ -702,7 +702,7 @@ static void launch_step(WalkArgs &a, int step, int64_t units, hipStream_t st)
     a.heavy_only = false;
     const int grid = (int)std::min<int64_t>(kWalkBlocks, (units + 2 * kXcds - 1) / (2 * kXcds) * (2 * kXcds));
     a.tile = units <= kWalkBlocks ? 2 : 64;
-    if (units <= kWideUnits || step == 0) {
+    if (units <= kWideUnits) {
         int2 *const heavy = a.heavy;
         a.heavy = nullptr;  // none put off
         k_walk_step<8, 4096, 4, STORE><<<grid, 512, 0, st>>>(a);
@@ -710,7 +710,7 @@ static void launch_step(WalkArgs &a, int step, int64_t units, hipStream_t st)
         return;
     }
     k_walk_step<2, 1920, 5, STORE><<<grid, 128, 0, st>>>(a);
-    if (!a.heavy) return;
+    if (!a.heavy || step == 0) return;  // (of the start targets none are put off)
     a.heavy_only = true;
     k_walk_step<12, 9408, 6, STORE><<<kHeavyBlocks, 768, 0, st>>>(a);
 }
