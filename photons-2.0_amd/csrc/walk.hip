@@ -814,15 +814,26 @@ void run_walk_from(Ctx &c, int shift_lo, int shift_hi, int start_target, int sta
         for (size_t k = 0; k < words; k++) cap[k / kCountSlots] += (int64_t)pin[k];
         make_room(held);
     };
-    for (int d = 0; d <= ndepth; d++) {
+    // a walk from a given cell: its children's depth is the next one with targets
+    int next = 1;
+    if (!forest) {
+        CellInfo *pin = reinterpret_cast<CellInfo *>(c.pinned.p);
+        PH_CHECK(hipMemcpyAsync(pin, dptr<CellInfo>(c.info) + start_target, sizeof(CellInfo), hipMemcpyDeviceToHost, st));
+        PH_CHECK(hipStreamSynchronize(st));
+        next = pin->depth + 1;
+    }
+    for (int d = 0; d <= ndepth; d = d == 0 ? next : d + 1) {
         const int64_t units = d == 0 ? nstart
                                      : 2 * std::min<int64_t>(nnb, d < 32 ? (int64_t)nstart << (d - 1) : (int64_t)nnb);
+        const int64_t down = cap[kDown];
         if (!planned) count_ahead([&] { launch_step<false>(a, d, units, st); });
         launch_step<true>(a, d, units, st);
+        if (!planned && cap[kDown] == down) break;  // nothing passed down: no targets below
     }
-    if (!planned)
-        count_ahead([&] { launch_step<false>(a, kLeaves, nlb, st); });
-    launch_step<true>(a, kLeaves, nlb, st);
+    if (planned || cap[kDown] > 0) {
+        if (!planned) count_ahead([&] { launch_step<false>(a, kLeaves, nlb, st); });
+        launch_step<true>(a, kLeaves, nlb, st);
+    }
     k_walk_end<<<1, 1, 0, st>>>(sz, a.st, cap[kP2P], cap[kM2L], cap[kDown]);
     if (!planned) {
         c.n_p2p = cap[kP2P];
