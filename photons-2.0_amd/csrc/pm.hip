@@ -502,32 +502,38 @@ int photons_pm_force_device(photons_pm *p, int64_t n, const double *d_pos, doubl
         PM_CHECK(rocprim::radix_sort_pairs(p->sort_tmp, tmp_bytes, kb, vb, (size_t)n, 0, bits, st));
         const uint32_t *skey = kb.current();
         const int32_t *sidx = vb.current();
-        if (n < kRowsParticles) {
+        // by rows: at most one run per mesh point, and one more per wavefront
+        const int nwave = blocks(n, 64);
+        const int64_t cap = std::min<int64_t>(n, (int64_t)n3 + nwave);
+        bool rows = n >= kRowsParticles;
+        size_t scan_bytes = 0, at_byte = 0;
+        if (rows)
+            PM_CHECK(rocprim::exclusive_scan(nullptr, scan_bytes, (int *)nullptr, (int *)nullptr, 0, (size_t)nwave,
+                                             rocprim::plus<int>(), st));
+        auto piece = [&](size_t bytes) {
+            const size_t b = at_byte;
+            at_byte += (bytes + 255) / 256 * 256;
+            return b;
+        };
+        const size_t o_sums = piece(sizeof(double2) * 4 * cap), o_key = piece(sizeof(uint32_t) * cap),
+                     o_count = piece(sizeof(int) * nwave), o_off = piece(sizeof(int) * nwave),
+                     o_row = piece(sizeof(int) * ((size_t)N * N + 1)), o_scan = piece(scan_bytes);
+        if (rows && at_byte > p->runs_bytes) {
+            if (p->runs) PM_CHECK(hipFree(p->runs));
+            p->runs = nullptr;
+            p->runs_bytes = 0;
+            if (hipMalloc(&p->runs, at_byte) == hipSuccess) {
+                p->runs_bytes = at_byte;
+            } else {  // (up to 68 bytes a particle: no memory left for them, by atomics then)
+                (void)hipGetLastError();
+                p->runs = nullptr;
+                rows = false;
+            }
+        }
+        if (!rows) {
             k_fill<<<blocks(n3, 256), 256, 0, st>>>(p->mesh, n3, 0.0);
             k_deposit_runs<<<blocks(n, 256), 256, 0, st>>>(n, d_pos, skey, sidx, p->mass, N, norm, delta, p->mesh);
         } else {
-            // at most one run per mesh point, and one more per wavefront
-            const int nwave = blocks(n, 64);
-            const int64_t cap = std::min<int64_t>(n, (int64_t)n3 + nwave);
-            size_t scan_bytes = 0;
-            PM_CHECK(rocprim::exclusive_scan(nullptr, scan_bytes, (int *)nullptr, (int *)nullptr, 0, (size_t)nwave,
-                                             rocprim::plus<int>(), st));
-            size_t at_byte = 0;
-            auto piece = [&](size_t bytes) {
-                const size_t b = at_byte;
-                at_byte += (bytes + 255) / 256 * 256;
-                return b;
-            };
-            const size_t o_sums = piece(sizeof(double2) * 4 * cap), o_key = piece(sizeof(uint32_t) * cap),
-                         o_count = piece(sizeof(int) * nwave), o_off = piece(sizeof(int) * nwave),
-                         o_row = piece(sizeof(int) * ((size_t)N * N + 1)), o_scan = piece(scan_bytes);
-            if (at_byte > p->runs_bytes) {
-                if (p->runs) PM_CHECK(hipFree(p->runs));
-                p->runs = nullptr;
-                p->runs_bytes = 0;
-                PM_CHECK(hipMalloc(&p->runs, at_byte));
-                p->runs_bytes = at_byte;
-            }
             char *w = static_cast<char *>(p->runs);
             double2 *sums = reinterpret_cast<double2 *>(w + o_sums);
             uint32_t *rkey = reinterpret_cast<uint32_t *>(w + o_key);
