@@ -596,11 +596,12 @@ constexpr int kSubThreads = 512;
 // levels, so that the largest segment counts and not the level.  Tree phase, by the level's
 // number against this: 2M particles with half of them in one clump 2.7 -> 1.2 ms (all levels by
 // chunks: 1.6), 2M with log-uniform radii over six decades 3.5 -> 1.3 (1.8), 256^3 clustered
-// ones 8.3 -> 7.1 (9.2).  A workgroup takes 2.1 us per 1000 particles, a level by chunks some 50 us and 0.25
-// ms at 256^3: limits of 8192, 16384, 32768, 65536 and 131072 give 6.5, 6.9, 7.4, 7.6 and 8.1 ms
-// there, 1.25, 1.25, 1.32, 1.42 and 1.57 at 128^3; replayed evaluations of 20,000 to 100,000
-// particles are within 1% from 12288 to 32768.
-constexpr int kWgSegment = 24576;
+// ones 8.3 -> 7.4 (9.2).  A workgroup takes 2.1 us per 1000 particles, a level by chunks some 50
+// us and 0.25 ms at 256^3: limits of 8192, 16384, 32768, 65536 and 131072 give 6.5, 6.9, 7.4, 7.6
+// and 8.1 ms there, 1.25, 1.25, 1.32, 1.42 and 1.57 at 128^3.  Planned evaluations of balanced
+// boxes lose by limits below 32768 (24576: 32^3 particles 620 -> 633 us, 1M uniform ones 6.53 ->
+// 6.58 ms).
+constexpr int kWgSegment = 32768;
 
 // Forests of more than kManyBoxes boxes of at most kFewLeaves leaves' worth of particles go
 // level by level: there are few levels, whereas each box costs its subtrees' workgroups some
