@@ -610,7 +610,7 @@ def main():
         "p2p_interactions": inter,
         "tree": {"nleaf": st["nleaf"], "nnode": st["nnode"], "depth": st["depth"],
                  "p2p_pairs": st["p2p_pairs"], "m2l_pairs": st["m2l_pairs"]},
-        "roofline": {"bound": "valu", "kernel": "k_p2p_table" if n >= 900000 or not fp32 else "k_p2p_f32", "achieved": achieved,
+        "roofline": {"bound": "valu", "kernel": "k_p2p_table (small FP32-mixed boxes: k_p2p_f32)", "achieved": achieved,
                      "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak,
                      "traffic": (P2P_FP32_TRAFFIC_256 if fp32 and args.nside == 256 and prm.order == 4 else None),
                      "note": "27 flops per interaction x interactions / mean P2P kernel time (HIP events on the "
