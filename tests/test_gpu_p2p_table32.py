@@ -56,3 +56,32 @@ def test_forces_match_the_direct_sum(maxleaf, soft_rs, order, mesh):
         bound = (f * per_pair).sum() + 4 * EPS * (np.sqrt(len(r)) + 64) * f.sum()
         err = np.linalg.norm(acc[s] - want[i])
         assert err <= bound, (i, err, bound, np.linalg.norm(want[i]))
+
+
+def test_forest_of_boxes_by_both_kernels():
+    """boxes on both sides of the limit in one evaluation: each as alone, bit for bit"""
+    import torch
+    counts = np.array([3000, N, 899999, 40000, 70])
+    lengths = 500000.0 * (counts / 256.0 ** 3) ** (1.0 / 3.0)
+    r = np.random.Generator(np.random.PCG64(7))
+    parts = [r.random((c, 3)) * L for c, L in zip(counts, lengths)]
+    prm = ic.force_params(256 ** 3, 500000.0, 256, rc_factor=6.0, theta=0.5, order=3).as_dict()
+    alone = []
+    for p, L in zip(parts, lengths):
+        ctx = pg.Context(dict(prm, boxsize=float(L)), pg.FP32_MIXED)
+        alone.append(ctx.force(p))
+        ctx.close()
+    want = np.concatenate(alone)
+    d_pos = torch.from_numpy(np.concatenate(parts)).cuda()
+    d_acc = torch.zeros_like(d_pos)
+    ctx = pg.Context(prm, pg.FP32_MIXED)
+    for again in range(2):  # ordinary, then planned
+        assert np.array_equal(ctx.force_boxes(counts, lengths, np.concatenate(parts)), want)
+    ctx.graph_create(counts, lengths, d_pos.data_ptr(), d_acc.data_ptr())
+    for rep in range(3):
+        d_acc.zero_()
+        torch.cuda.synchronize()
+        ctx.graph_launch()
+        assert ctx.graph_check()[0] == 0
+        assert np.array_equal(d_acc.cpu().numpy(), want), rep
+    ctx.close()
