@@ -44,7 +44,7 @@ P2P_FLOPS = 27  # per particle-particle interaction
 # HBM bytes per FP32 P2P launch (k_p2p_table<float, 4>) at 256^3 clustered, p = 4, from
 # rocprofv3 --pmc FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 (factors from a 1 GiB copy in the
 # same run); the counts and commands are kept with the P2P counter summary under profiles/
-P2P_FP32_TRAFFIC_256 = (2.0 * 65201137 + 1410868) * 1024
+P2P_FP32_TRAFFIC_256 = (2.0 * 65729600 + 1411190) * 1024
 
 
 def log(msg):
@@ -615,7 +615,7 @@ def main():
                      "traffic": (P2P_FP32_TRAFFIC_256 if fp32 and args.nside == 256 and prm.order == 4 else None),
                      "note": "27 flops per interaction x interactions / mean P2P kernel time (HIP events on the "
                              "library's stream); bound by the LDS (a table row per interaction, read at random) "
-                             "and the vector ALU (19 instructions per FP32 interaction) at once; packed FP32 is "
+                             "and the vector ALU (21 instructions per FP32 interaction) at once; packed FP32 is "
                              "not used, so 78.6 of the 157.3 TFLOP/s peak is reachable at most; traffic = HBM "
                              "bytes per launch from rocprofv3 PMC"},
     }

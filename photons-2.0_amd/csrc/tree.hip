@@ -587,7 +587,7 @@ __global__ void k_emit_leaves(const DevSizes *__restrict__ sz, const int *__rest
 // so that only the top of the tree goes level by level, with segments of up to
 // kWgSegment particles split by one workgroup each in one launch (k_split_level).
 // Measured, tree phase: 16^3 particles 0.60 -> 0.12 ms, 64^3 0.96 -> 0.52 ms, 100k in leaves
-// of 8 1.10 -> 0.34 ms, 256^3 9.5 -> 8.1 ms (there the passes of the top levels remain).
+// of 8 1.10 -> 0.34 ms, 256^3 9.5 -> 7.3 ms (there the passes of the top levels remain).
 constexpr int kSubtree = 1024;     // particles of a stem, at leaves of 8 and more
 constexpr int kSubNodes = 512;     // nodes of a subtree (leaves: one more)
 constexpr int kSubThreads = 512;

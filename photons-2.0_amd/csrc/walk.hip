@@ -358,10 +358,11 @@ __device__ __forceinline__ int64_t take(const WalkArgs &a, int list, int64_t n)
 //
 // What bounds it: a box of few cells, the chain of dependent loads and barriers of one step
 // (12 us) times the depths; a large one, latency too: 65% of the wavefronts' cycles are
-// waits, at 24 wavefronts per CU (LDS).  Against the walk it replaces (two passes over the
+// waits.  The windows leave a CU 18 wavefronts of the narrow workgroups (17 KB each) and 24 of
+// the wide ones (two of half the LDS).  Against the walk it replaces (two passes over the
 // traversals of single lanes, a dozen launches per depth): 16^3 clustered particles 0.68 ->
-// 0.20 ms, 64^3 1.56 -> 0.65, 10^6 uniform ones 1.39 -> 0.6, 128^3 clustered 6.1 -> 4.0,
-// 256^3 35.8 -> 24.3 ms.
+// 0.20 ms, 64^3 1.56 -> 0.71, 10^6 uniform ones 1.39 -> 0.65, 128^3 clustered 6.1 -> 3.3, 256^3
+// 35.8 -> 23.1 ms.
 template <int NW, int CAP, int EU, bool STORE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(EU))) k_walk_step(WalkArgs a)
 {
