@@ -13,7 +13,9 @@
 //   * lam^2 = (2^(j+1) - 2) / eps^2, so that r = eps, where F has a kink, is the start of
 //     a row; j >= 1 is the smallest for which the first row (s in [2, 2 + 1/32)) resolves
 //     the u^3 of G near 0, which is not smooth in s (u at s - 2 = 2: at most kUMin);
-//   * rows end at r = u_end 2 rs; the last one is zero.
+//   * rows end with the octave of r = u_end 2 rs, in FP64 at u = 8.7 at most, where they are
+//     off by 9e-9 (G = 2e-32); the last one is zero.  (Ending at u = 8 costs: each batch with a pair beyond
+//     the table is gone through again; 1M uniform particles 11.6 -> 12.6 ms, 256^3 248 -> 250.)
 //
 //             rows/octave  row                                   u up to   relative error of F
 //   FP32      64           4 floats, cubic in s - s_mid          9.5       2e-7 (u < 1), 4e-7 (u < 3)
@@ -34,6 +36,7 @@
 // Plain C++, so that it can be tested on the host.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -54,7 +57,7 @@ constexpr int kPairBits32 = 6, kPairBits64 = 6;  // rows per octave: 2^bits
 // octaves at most (the row index takes the five low exponent bits): the FP64 rows, 3 KB
 // per octave, share a workgroup's LDS with the staged particles
 constexpr int kPairOctaves = 31;
-constexpr double kPairUEnd32 = 9.5, kPairUEnd64 = 8.0;
+constexpr double kPairUEnd32 = 9.5, kPairUEnd64 = 8.0, kPairUMost64 = 8.7;
 constexpr double kPairUMin32 = 0.06, kPairUMin64 = 3.5e-4;
 
 #ifdef __HIPCC__
@@ -93,6 +96,13 @@ inline PairShape pair_shape(double eps, double rs, bool f32)
     if (t.octaves < j) t.octaves = j;  // eps beyond the end of the split factor
     if (t.octaves > kPairOctaves) return t;
     t.rows = (t.octaves << (f32 ? kPairBits32 : kPairBits64)) + 1;
+    if (!f32) {  // the octave may go on to u = 11.3, where the rows are off by some 1e-7
+        const double most = kPairUMost64 * 2.0 * rs * t.lam, s = most * most + 2.0;
+        uint64_t b;
+        std::memcpy(&b, &s, 8);
+        const int row = (int)((uint32_t)(b >> 32) - (1024u << 20)) >> (20 - kPairBits64);
+        t.rows = std::min(t.rows, std::max(row + 1, j << kPairBits64) + 1);
+    }
     return t;
 }
 
@@ -168,6 +178,9 @@ PAIR_HD inline PairRow64 pair_row64(int i, int rows, double lam2, double eps, do
     return R;
 }
 
+// the high word of s from which on the FP64 rows end
+inline uint32_t pair_top64(int rows) { return (1024u << 20) + ((uint32_t)(rows - 1) << (20 - kPairBits64)); }
+
 // the table on the host (for tests; the library's is built on the device, row by row)
 struct PairTable : PairShape {
     bool valid = false;
@@ -210,7 +223,7 @@ inline double pair_eval64(const PairTable &t, double r)
     const double s = std::fma(r * r, t.lam2, 2.0);
     uint64_t b;
     std::memcpy(&b, &s, 8);
-    const uint32_t hi = (uint32_t)(b >> 32), top = (uint32_t)(1024 + t.octaves) << 20;
+    const uint32_t hi = (uint32_t)(b >> 32), top = pair_top64(t.rows);
     if (hi >= top) return 0.0;  // the kernels evaluate the factor itself from there on
     const uint64_t xm = ((uint64_t)((hi & 0xfffffu) | 0x3ff00000u) << 32) | (b & 0xffffffffu);
     const uint64_t xc = (uint64_t)((hi & 0xfc000u) | 0x3ff02000u) << 32;
